@@ -1,6 +1,6 @@
-"""The large-grid attention kernel (attn_fwd_d64) where its fp16-pair and fp32
-paths meet: sequence ends inside a key tile and a query block, every mask form,
-and operands that fp16 cannot hold; and the grids around its least size."""
+"""The large-grid attention kernel (attn_fwd_d64) where its 16-bit and fp32 matrix
+paths meet: sequence ends inside a key tile and a query block, every mask form, and
+operands that the 16-bit forms cannot hold; and the grids around its least size."""
 import ctypes as C
 
 import numpy as np
@@ -30,7 +30,8 @@ def _run(ctx, q, k, v, mask, fill, off=0):
     return out.numpy()
 
 
-def _ref(q, k, v, mask, fill):
+def _ref(q, k, v, mask, fill, magnitude=False):
+    """In 64 bits; magnitude: sum of the weights times |v| instead."""
     B, S, H = q.shape
     n = H // HD
     hd = lambda a: a.astype(np.float64).reshape(B, S, n, HD).transpose(0, 2, 1, 3)  # noqa: E731
@@ -38,7 +39,7 @@ def _ref(q, k, v, mask, fill):
     if mask is not None:
         s = np.where(np.broadcast_to(mask, s.shape), np.float64(np.float32(fill)), s)
     p = np.exp(s - s.max(-1, keepdims=True))
-    o = (p / p.sum(-1, keepdims=True)) @ hd(v)
+    o = (p / p.sum(-1, keepdims=True)) @ (np.abs(hd(v)) if magnitude else hd(v))
     return o.transpose(0, 2, 1, 3).reshape(B, S, H)
 
 
@@ -76,8 +77,9 @@ def test_attention_tiles_masks_and_edges(ctx, S, B, form):
 
 
 @pytest.mark.parametrize("S,B,heads", [(100, 26, 12), (200, 13, 12)])
-@pytest.mark.parametrize("kind", ["tiny_v", "tiny_qk", "zero_v", "sharp", "late_max", "huge_v",
-                                  "huge_masked", "soft_fill"])
+@pytest.mark.parametrize("kind", ["tiny_v", "subnormal_v", "tiny_qk", "zero_v", "sharp",
+                                  "late_max", "huge_v", "huge_masked", "soft_fill", "large_qk",
+                                  "masked_large_v", "small_late_v", "mixed_v", "one_key"])
 def test_attention_tiles_operand_ranges(ctx, S, B, heads, kind):
     q, k, v = _inputs(B, S, heads, len(kind))
     lens = np.random.default_rng(3).integers(max(1, S // 4), S + 1, B)
@@ -86,6 +88,8 @@ def test_attention_tiles_operand_ranges(ctx, S, B, heads, kind):
     fill = graphs.FILL_MIN
     if kind == "tiny_v":
         v *= np.float32(1e-9)
+    elif kind == "subnormal_v":
+        v *= np.float32(1e-39)
     elif kind == "tiny_qk":
         q *= np.float32(1e-5)
         k *= np.float32(1e-5)
@@ -104,11 +108,40 @@ def test_attention_tiles_operand_ranges(ctx, S, B, heads, kind):
     elif kind == "soft_fill":  # masked keys keep a weight
         fill = -2.5
         mask = np.random.default_rng(4).random((B, 1, S, S)) < 0.4
+    elif kind == "large_qk":  # small elements of q meet large ones of k
+        q *= np.float32(1e-6)
+        k *= np.float32(1e5)
+    elif kind == "masked_large_v":  # the first keys are masked and large, the rest small
+        mask[..., :40] = True
+        lens = np.maximum(lens, 60)
+        mask[..., 40:] = np.arange(40, S)[None, :] >= lens[:, None, None, None]
+        v[:, 40:] *= np.float32(1e-12)
+    elif kind == "small_late_v":  # the same, the first keys unmasked but without weight
+        k[..., :40, :] = -50.0 * np.sign(q[:, :1])
+        q[:] = np.abs(q) * np.sign(q[:, :1])
+        k[:, 40:] *= np.float32(0.1)
+        v[:, 40:] *= np.float32(1e-12)
+    elif kind == "mixed_v":  # every dim spans many decades
+        v *= np.float32(10.0) ** np.random.default_rng(6).uniform(-30, 10, v.shape).astype(np.float32)
+    elif kind == "one_key":  # each query all but selects one key
+        k[:] = 0.0
+        for d in range(HD):
+            k[:, d::HD, d::HD] = 60.0
+        q[:] = 0.0
+        pick = np.random.default_rng(7).integers(0, HD, (B, S, heads))
+        np.put_along_axis(q.reshape(B, S, heads, HD), pick[..., None], np.float32(8.0), -1)
+        v *= np.float32(10.0) ** np.random.default_rng(8).uniform(-20, 0, v.shape).astype(np.float32)
     got, ref = _run(ctx, q, k, v, mask, fill), _ref(q, k, v, mask, fill)
     assert np.isfinite(got).all()
-    # per (text, dim): the largest |v| of that dim bounds its outputs
-    top = np.abs(v).max(1, keepdims=True) + 1e-30
-    assert (np.abs(got - ref) / top).max() <= (3e-5 if kind in ("sharp", "late_max") else 1e-5)
+    # Every output against its own terms, sum p |v|: the scores' rounding (64 products at
+    # 2^-24 of their sum of magnitudes) is a relative error of the weights, as are the
+    # rounding of S weights' sums; half a subnormal step where the terms are that small.
+    d = lambda a: a.astype(np.float64).reshape(B, S, heads, HD).transpose(0, 2, 1, 3)  # noqa: E731
+    scores = (np.abs(d(q)) @ np.abs(d(k)).transpose(0, 1, 3, 2)).max() / 8.0
+    lim = 2.0 ** -23 * scores + S * 2.0 ** -24
+    mag = _ref(q, k, v, mask, fill, magnitude=True)
+    assert (np.abs(got - ref) <= lim * mag + 2.0 ** -149).all(), \
+        float((np.abs(got - ref) / (mag + 1e-300)).max() / lim)
 
 
 @pytest.mark.parametrize("S,B", [(120, 260), (180, 140)])
