@@ -75,6 +75,23 @@ def test_gemm_small_m_edges(ctx, tb, M, N, K):
     _check(_run(ctx, a, b, 0, tb), a, b)
 
 
+# few tiles: K goes over as many blocks as there are CUs, in splits of 192 at least
+@pytest.mark.parametrize("ta,tb,M,N,K", [
+    (0, 0, 1, 3, 575), (0, 0, 1, 3, 576), (0, 0, 64, 63, 1500), (1, 0, 100, 200, 1501),
+    (0, 0, 600, 256, 1000), (0, 1, 513, 129, 2049), (1, 1, 512, 512, 769), (0, 0, 65, 63, 20000)])
+def test_gemm_few_tiles_split_k(ctx, ta, tb, M, N, K):
+    rng = np.random.default_rng(M + N + K)
+    a = rng.standard_normal((M, K)).astype(np.float32)
+    b = (0.02 * rng.standard_normal((K, N))).astype(np.float32)
+    c = rng.standard_normal(N).astype(np.float32)
+    got = _run(ctx, a, b, ta, tb, c)
+    # (the sum with C rounds once more, at 2^-24 of an output)
+    err = np.abs(got - (a.astype(np.float64) @ b + c))
+    mag = np.abs(a).astype(np.float64) @ np.abs(b) + np.abs(c)
+    assert (err <= (2.0 ** -21 + 3 * K * 2.0 ** -24) * mag).all()
+    np.testing.assert_array_equal(_run(ctx, a, b, ta, tb, c), got)
+
+
 VALUES = ["tiny_a", "tiny_b", "zero_row", "late_row", "huge", "mixed", "subnormal", "integers",
           "one_hot"]
 

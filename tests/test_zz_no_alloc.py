@@ -16,8 +16,8 @@ from inferc_amd.rt import Tensor
 
 pytestmark = pytest.mark.gpu
 
-# (transA, M, N, K): split-K with 16 splits (M > 512, the small-M kernel
-# cannot take it), then a smaller one with 16, then transA with 23 splits
+# (transA, M, N, K): split-K with 6 splits on 256 CUs (M > 512, the small-M kernel
+# cannot take it), then a smaller product with 10, then transA with 15 splits
 SHAPES = [(0, 600, 256, 4096), (0, 520, 128, 2048), (1, 100, 200, 3000)]
 
 
