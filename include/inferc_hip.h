@@ -145,6 +145,17 @@ int inferc_hip_gemm_f32_noalloc(inferc_hip_ctx* ctx, int trans_a, int trans_b,
                                 int c_kind, int64_t ldc, const float* R,
                                 int64_t ldr, int act, float* Y, int64_t ldy);
 
+/* Which kernel a dense product of these sizes runs on a device of num_cus compute units,
+ * and how its K is split (host only; no context, no device). aligned: 16-byte aligned
+ * operands whose contiguous extents and leading dimensions are multiples of 4. plan:
+ * [0], [1] rows and columns of an output tile, [2] blocks sharing a tile's K, [3] K groups
+ * in a block of the LDS-tiled kernel, 0 for the small-M kernel, [4], [5] the former's grid
+ * of tiles, x and z. The one-row GEMV route (src/kernels/matmul.cc:207-216) is not
+ * covered. For tests of the dispatch and for planning; the choice may change. */
+int inferc_hip_gemm_plan(int trans_a, int trans_b, int64_t M, int64_t N,
+                         int64_t K, int64_t batch, int aligned, int num_cus,
+                         int64_t* plan);
+
 /* numpy MatMul over a flattened batch: Y[b] = A[b*stride_a] * B[b*stride_b],
  * a stride of 0 broadcasts. Replaces rt::MatMul, src/kernels/matmul.cc:63-159. */
 int inferc_hip_matmul_f32(inferc_hip_ctx* ctx, int64_t batch, int64_t M,

@@ -1,0 +1,41 @@
+"""The dispatch of dense products (inferc_hip_gemm_plan, host only): the K split, and the
+grid of the widest products."""
+from __future__ import annotations
+
+import ctypes as C
+
+import pytest
+
+from inferc_amd import lib as L
+
+CUS = 256  # MI355X
+
+
+def plan(M, N, K, ta=0, tb=0, batch=1, cus=CUS):
+    out = (C.c_int64 * 6)()
+    aligned = (M if ta else K) % 4 == 0 and (K if tb else N) % 4 == 0
+    L.check(L.load_library().inferc_hip_gemm_plan(ta, tb, M, N, K, batch, int(aligned), cus, out))
+    return dict(zip(("rows", "cols", "splits", "groups", "x", "z"), out))
+
+
+def form(*shape, **kw):
+    p = plan(*shape, **kw)
+    return "small" if p["groups"] == 0 else f"{p['rows']}x{p['groups']}"
+
+
+def test_few_tiles_split_k():
+    assert plan(64, 63, 1500)["splits"] == 7 and plan(64, 63, 575)["splits"] == 1
+    assert plan(600, 256, 1000)["splits"] == 5  # 40 tiles
+    assert plan(700, 700, 768)["splits"] == 1  # 121 tiles: no CU is idle
+    assert plan(512, 768, 3072, tb=1)["splits"] == 4
+
+
+@pytest.mark.parametrize("M,N", [(1, 2 ** 31 - 65), (64, 2 ** 30 + 1), (100, 2 ** 31 - 65),
+                                 (128, 2 ** 30 + 77), (4096, 3072), (4 * 10 ** 6, 65)])
+def test_grid_dimensions_stay_below_2_32_threads(M, N):
+    """One K and 2^30 columns and more: accepted, so the grid has to hold the tiles."""
+    p = plan(M, N, 1)
+    threads = 256 if (p["rows"], p["groups"]) == (64, 1) else 512
+    tiles = -(-M // p["rows"]) * -(-N // p["cols"])
+    assert p["x"] * threads < 2 ** 32 and p["x"] * p["z"] >= tiles > p["x"] * (p["z"] - 1)
+    assert p["z"] < 65536
