@@ -1,5 +1,5 @@
-"""The dispatch of dense products (inferc_hip_gemm_plan, host only): the K split, and the
-grid of the widest products."""
+"""The dispatch of dense products (inferc_hip_gemm_plan, host only): that the shapes of
+the GPU tests run the kernels they are there for, and the grid of the widest products."""
 from __future__ import annotations
 
 import ctypes as C
@@ -7,6 +7,7 @@ import ctypes as C
 import pytest
 
 from inferc_amd import lib as L
+from tests import test_gpu_gemm_tile as T
 
 CUS = 256  # MI355X
 
@@ -21,6 +22,33 @@ def plan(M, N, K, ta=0, tb=0, batch=1, cus=CUS):
 def form(*shape, **kw):
     p = plan(*shape, **kw)
     return "small" if p["groups"] == 0 else f"{p['rows']}x{p['groups']}"
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_edge_shapes_run_the_tiles_they_name(ta, tb):
+    forms = [form(*s, ta=ta, tb=tb) for s in T.EDGES_64]
+    assert set(forms) == {"64x1", "64x2"}
+    assert {form(*s, ta=ta, tb=tb) for s in T.EDGES_128} == {"128x1"}
+    # K below, at and above the fp16 path's least K, whole and ragged panels
+    assert any(s[2] < 64 for s in T.EDGES_128) and any(s[2] > 64 for s in T.EDGES_128)
+    assert any(s[2] == 64 for s in T.EDGES_128)
+
+
+def test_small_m_shapes_run_every_form():
+    got = {tuple(list(plan(*s, tb=tb).values())[:4]) for s in T.SMALL for tb in (0, 1)}
+    small = {g[:3] for g in got if g[3] == 0}
+    assert small == {(16, 16, 1), (16, 32, 1), (16, 48, 2), (32, 48, 1), (32, 64, 1)}
+    assert any(g[3] == 2 for g in got)  # the tiles that replace them
+
+
+def test_value_shapes_reach_every_kernel():
+    for shapes in (T.RANGES, T.MEETS):
+        got = {form(*s, tb=tb) for s in shapes for tb in (0, 1)}
+        assert {"small", "64x2", "128x1"} <= got
+    assert {form(M, N, 160, ta=ta, tb=tb) for ta, tb, M, N in T.INFINITIES} >= {
+        "small", "64x2", "128x1"}
+    assert {form(*s) for s in T.EPILOGUES} >= {"64x2", "64x1", "128x1"}
+    assert any(form(*s) == "128x1" and s[2] < 64 for s in T.EPILOGUES)
 
 
 def test_few_tiles_split_k():

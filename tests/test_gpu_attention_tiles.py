@@ -8,6 +8,7 @@ import pytest
 
 from inferc_amd import graphs, lib as L, rt
 from inferc_amd.rt import Tensor
+from tests import ref64
 
 pytestmark = pytest.mark.gpu
 HD = 64
@@ -74,6 +75,37 @@ def test_attention_tiles_masks_and_edges(ctx, S, B, form):
     for off in (0, 1):
         _close(_run(ctx, q, k, v, mask, graphs.FILL_MIN, off),
                _ref(q, k, v, mask, graphs.FILL_MIN), v)
+
+
+# the large-grid kernel starts at 256 blocks of 128 queries (one a CU), at 128 for four key
+# tiles and more: the last grid of the small-grid kernels and the first of it
+@pytest.mark.parametrize("S,B", [(96, 255), (96, 256), (97, 127), (97, 128), (97, 255), (200, 63),
+                                 (200, 64), (200, 127), (300, 42), (300, 43)])
+@pytest.mark.parametrize("form", ["none", "row"])
+def test_attention_grids_around_the_least_size(ctx, S, B, form):
+    q, k, v = _inputs(B, S, 1, S * B)
+    mask = None
+    if form == "row":
+        lens = np.random.default_rng(B).integers(1, S + 1, B)
+        mask = (np.arange(S)[None, :] >= lens[:, None]).reshape(B, 1, 1, S)
+    _close(_run(ctx, q, k, v, mask, graphs.FILL_MIN), _ref(q, k, v, mask, graphs.FILL_MIN), v)
+
+
+@pytest.mark.parametrize("n", [896, 897, 1000, 1024, 1051])
+def test_attention_tiles_causal_prefill(ctx, n):
+    """A causal prefill of 16 heads: 112 blocks (small-grid kernel) at 896 tokens, 128 and
+    more (the large-grid kernel's causal rule, tile skip and score masks) from 897. The
+    queries and keys are large, so that a key more or less moves the logits by 1e-2."""
+    cfg = dict(layers=1, hidden=1024, heads=16, ffn=128, vocab=200, max_pos=1051, eps=1e-5)
+    w = graphs.gpt2_weights(cfg, 11)
+    w[4] = (w[4] * np.float32(4)).astype(np.float32)  # QKV
+    w[6] = (w[6] * np.float32(4)).astype(np.float32)  # out-projection
+    ids = np.random.default_rng(n).integers(0, cfg["vocab"], n)
+    dec = rt.Gpt2Decoder(ctx, cfg, w, max_t=cfg["max_pos"])
+    got = dec.forward(ids)
+    dec.close()
+    ref = ref64.gpt2_logits(cfg, w, ids)
+    assert np.abs(got - ref).max() <= 1e-4, float(np.abs(got - ref).max())
 
 
 @pytest.mark.parametrize("S,B,heads", [(100, 26, 12), (200, 13, 12)])

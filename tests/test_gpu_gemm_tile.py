@@ -2,7 +2,8 @@
 the sizes and operand values where their two paths, fp16 pairs and plain fp32
 products, meet: K around a panel and around the fp16 path's least K, ragged
 tiles of every form, every orientation, and operands below, above and outside
-fp16's range."""
+fp16's range. Which kernel the shapes run on 256 CUs is checked, without a GPU, by
+test_gemm_plan.py."""
 import ctypes as C
 
 import numpy as np
@@ -48,11 +49,16 @@ def _check(got, a, b):
 
 
 # M > 512 keeps the small-M kernel away; the tile forms' edges are 64 and 128
+EDGES_64 = [(513, 1, 1), (513, 65, 31), (576, 63, 32), (640, 129, 33), (515, 64, 63),
+            (520, 68, 64), (519, 130, 65), (1000, 257, 96), (513, 384, 1536), (514, 131, 1601),
+            (4097, 1025, 68), (4100, 1100, 40), (70, 40001, 65), (40000, 66, 96)]
+EDGES_128 = [(5120, 1280, 128), (2000, 2000, 130), (1921, 2047, 1), (2047, 1921, 31),
+             (2001, 1999, 45), (1990, 2011, 63), (1985, 1985, 64), (2033, 1987, 97),
+             (100, 50257, 40)]
+
+
 @pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
-@pytest.mark.parametrize("M,N,K", [
-    (513, 1, 1), (513, 65, 31), (576, 63, 32), (640, 129, 33), (515, 64, 63), (520, 68, 64),
-    (519, 130, 65), (1000, 257, 96), (513, 384, 1536), (514, 131, 1601), (4097, 1025, 68),
-    (5120, 1280, 128)])
+@pytest.mark.parametrize("M,N,K", EDGES_64 + EDGES_128)
 def test_gemm_tile_edges(ctx, ta, tb, M, N, K):
     rng = np.random.default_rng(M * 7 + N * 3 + K + 2 * ta + tb)
     a = rng.standard_normal((M, K)).astype(np.float32)
@@ -63,11 +69,13 @@ def test_gemm_tile_edges(ctx, ta, tb, M, N, K):
 # M <= 512 with whole float4 rows: every form of the small-M kernel (16x16,
 # 16x32, 16x48 over two blocks, 32x64, 32x48) and the tiles that replace it
 # from two or three rounds of blocks up
+SMALL = [(2, 4, 4), (33, 64, 60), (31, 768, 64), (17, 132, 68), (97, 772, 100), (130, 1540, 96),
+         (130, 1732, 96), (128, 768, 3072), (100, 768, 2052), (255, 2304, 288), (129, 3072, 772), (300, 2308, 768),
+         (512, 3072, 768), (131, 768, 2048)]
+
+
 @pytest.mark.parametrize("tb", [0, 1])
-@pytest.mark.parametrize("M,N,K", [
-    (2, 4, 4), (33, 64, 60), (31, 768, 64), (17, 132, 68), (97, 772, 100), (130, 1540, 96),
-    (128, 768, 3072), (100, 768, 2052), (255, 2304, 288), (129, 3072, 772), (300, 2308, 768),
-    (512, 3072, 768), (131, 768, 2048)])
+@pytest.mark.parametrize("M,N,K", SMALL)
 def test_gemm_small_m_edges(ctx, tb, M, N, K):
     rng = np.random.default_rng(M * 7 + N * 3 + K + tb)
     a = rng.standard_normal((M, K)).astype(np.float32)
@@ -92,14 +100,16 @@ def test_gemm_few_tiles_split_k(ctx, ta, tb, M, N, K):
     np.testing.assert_array_equal(_run(ctx, a, b, ta, tb, c), got)
 
 
+RANGES = [(600, 200, 192), (4224, 1100, 100), (70, 200, 384), (128, 768, 3072),
+          (2000, 2010, 100)]
 VALUES = ["tiny_a", "tiny_b", "zero_row", "late_row", "huge", "mixed", "subnormal", "integers",
           "one_hot"]
 
 
 @pytest.mark.parametrize("kind", VALUES)
-@pytest.mark.parametrize("M,N,K", [(600, 200, 192), (4224, 1100, 100), (70, 200, 384),
-                                   (128, 768, 3072)])
-def test_gemm_tile_operand_ranges(ctx, M, N, K, kind):
+@pytest.mark.parametrize("tb", [0, 1])
+@pytest.mark.parametrize("M,N,K", RANGES)
+def test_gemm_tile_operand_ranges(ctx, M, N, K, kind, tb):
     rng = np.random.default_rng(len(kind) * 31 + M)
     a = rng.standard_normal((M, K)).astype(np.float32)
     b = (0.02 * rng.standard_normal((K, N))).astype(np.float32)
@@ -128,15 +138,17 @@ def test_gemm_tile_operand_ranges(ctx, M, N, K, kind):
     elif kind == "one_hot":
         a = np.eye(M, K, dtype=np.float32)
         a[K:, 0] = 1.0
-    got = _run(ctx, a, b, 0, 0)
+    got = _run(ctx, a, b, 0, tb)
     _check(got, a, b)
     if kind in ("integers", "one_hot"):  # exact in fp32 whatever the order
         np.testing.assert_array_equal(got, (a.astype(np.float64) @ b).astype(np.float32))
 
 
+MEETS = [(128, 768, 768), (600, 200, 768), (2, 64, 128), (4000, 3072, 96), (77, 50257, 96)]
+
+
 @pytest.mark.parametrize("tb", [0, 1])
-@pytest.mark.parametrize("M,N,K", [(128, 768, 768), (600, 200, 768), (2, 64, 128),
-                                   (4000, 3072, 96), (77, 50257, 96)])
+@pytest.mark.parametrize("M,N,K", MEETS)
 @pytest.mark.parametrize("pattern", ["block", "checker", "late", "columns"])
 def test_gemm_large_elements_meet_zeros(ctx, tb, M, N, K, pattern):
     """Outputs made of small elements alone, beside large ones that meet zeros of the
@@ -174,7 +186,8 @@ def test_gemm_large_elements_meet_zeros(ctx, tb, M, N, K, pattern):
 
 
 @pytest.mark.parametrize("ta", [0, 1])
-@pytest.mark.parametrize("M,N,K", [(600, 200, 768), (4000, 3072, 512), (128, 768, 768)])
+@pytest.mark.parametrize("M,N,K", [(600, 200, 768), (2000, 2003, 512), (4000, 3072, 512),
+                                   (128, 768, 768)])
 def test_gemm_zero_rows_that_stay_zero_or_not(ctx, M, N, K, ta):
     """Rows of A and columns of B that are zero over the first panel: over all of K, or
     with one element near the end (in the tiles, the former keep the fp16 path and the
@@ -193,10 +206,14 @@ def test_gemm_zero_rows_that_stay_zero_or_not(ctx, M, N, K, ta):
     assert np.abs(got[10] - want).max() <= 2.0 ** -22 * np.abs(want).max()
 
 
-@pytest.mark.parametrize("ta,tb,N", [(0, 0, 333), (1, 1, 333), (0, 1, 332)])
-def test_gemm_tile_infinities_and_nan(ctx, ta, tb, N):
-    """(N = 332 with 500 rows: the small-M kernel)"""
-    M, K = 777 if N == 333 else 500, 160
+INFINITIES = [(0, 0, 777, 333), (1, 1, 777, 333), (0, 1, 500, 332), (0, 0, 2000, 2003),
+              (0, 1, 2000, 2003), (1, 0, 2000, 2003)]
+
+
+@pytest.mark.parametrize("ta,tb,M,N", INFINITIES)
+def test_gemm_tile_infinities_and_nan(ctx, ta, tb, M, N):
+    """(N = 332 with 500 rows: the small-M kernel; 2000 rows: 128x128 tiles)"""
+    K = 160
     rng = np.random.default_rng(9)
     a = rng.standard_normal((M, K)).astype(np.float32)
     b = rng.standard_normal((K, N)).astype(np.float32)
@@ -215,10 +232,13 @@ def test_gemm_tile_infinities_and_nan(ctx, ta, tb, N):
     assert np.abs(got[ok] - ref[ok]).max() <= 1e-3
 
 
+EPILOGUES = [(530, 70, 96), (4200, 1000, 96), (2000, 1990, 96), (1990, 2001, 40)]
+
+
 def test_gemm_tile_residual_c_and_activation(ctx):
-    """The epilogue over ragged tiles of both forms: full C, residual, GELU."""
+    """The epilogue over ragged tiles of every form: full C, residual, GELU."""
     from math import erf
-    for M, N, K in [(530, 70, 96), (4200, 1000, 96)]:
+    for M, N, K in EPILOGUES:
         rng = np.random.default_rng(M)
         a = rng.standard_normal((M, K)).astype(np.float32)
         b = (0.1 * rng.standard_normal((K, N))).astype(np.float32)

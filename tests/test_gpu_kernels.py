@@ -190,8 +190,7 @@ def test_gemm_single_row_transb_epilogues(ctx, N, K):
 
 
 # Large-M products on the tiled kernel, with edge tiles (M, N not multiples
-# of the tile) and partial last K panels: 128x96 tiles (N % 96 == 0), 128x128
-# (N % 96 != 0, >= 3 tiles per CU), 128x64 (1-3 tiles per CU).
+# of the tile) and partial last K panels: 128x128 tiles, and 64x64 ones (N = 768).
 @pytest.mark.parametrize("M,N,K", [(4000, 768, 768), (4000, 3072, 100), (4032, 768, 45),
                                    (4000, 3136, 96), (2000, 2000, 130)])
 @pytest.mark.parametrize("act", [L.ACT_NONE, L.ACT_GELU_ERF])
