@@ -16,8 +16,9 @@ calibration (counter KiB that a copy of known size reads), and prints every
 other kernel's mean per-dispatch HBM bytes scaled by that factor.
 
 The ``--mfma`` form reads one ``rocprofv3 --pmc SQ_INSTS_VALU_MFMA_MOPS_F32
-SQ_VALU_MFMA_BUSY_CYCLES GRBM_GUI_ACTIVE`` CSV and prints per (kernel, grid):
-the fp32 MFMA FLOPs the counter saw (MOPS x 512) per dispatch, the dispatch's
+SQ_INSTS_VALU_MFMA_MOPS_F16 SQ_INSTS_VALU_MFMA_MOPS_BF16 SQ_VALU_MFMA_BUSY_CYCLES
+GRBM_GUI_ACTIVE`` CSV and prints per (kernel, grid): the MFMA FLOPs of the types
+counted (MOPS x 512; a product of fp16 pairs is three) per dispatch, the dispatch's
 duration (its timestamps) and the FLOP rate over it, the MFMA busy fraction
 SQ_VALU_MFMA_BUSY_CYCLES / (simds x GRBM_GUI_ACTIVE / xcc) (the busy counter
 is summed over every SIMD, the GUI counter over every XCC), the same busy
@@ -114,14 +115,15 @@ def mfma(path: str, simds: int, xcc: int, clock_mhz: float) -> list[dict]:
     groups = defaultdict(list)
     for (name, grid), ds in per.items():
         for d in ds.values():
-            fl = 512.0 * d.get("SQ_INSTS_VALU_MFMA_MOPS_F32", 0.0)
+            fl = d["flops"] = 512.0 * sum(v for k, v in d.items()
+                                          if k.startswith("SQ_INSTS_VALU_MFMA_MOPS_"))
             groups[(name, grid, float(f"{fl:.3e}"))].append(d)
     out = []
     for (name, grid, _), ds in groups.items():
         n = len(ds)
         mean = lambda k: sum(d.get(k, 0.0) for d in ds) / n  # noqa: E731
         us, gui = mean("us"), mean("GRBM_GUI_ACTIVE")
-        flops = 512.0 * mean("SQ_INSTS_VALU_MFMA_MOPS_F32")
+        flops = mean("flops")
         busy = mean("SQ_VALU_MFMA_BUSY_CYCLES")
         cyc = gui / xcc
         out.append({"kernel": name, "grid": grid, "dispatches": n, "us": us, "flops": flops,
