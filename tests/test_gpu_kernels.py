@@ -377,6 +377,20 @@ def test_activations_and_add(ctx):
     np.testing.assert_array_equal(rt.Add(T(ctx, row), T(ctx, a)).numpy(), a + row)
 
 
+@pytest.mark.parametrize("std,lim", [(1.0, 3.9e-8), (3.0, 3.0e-8), (6.0, 1.5e-8)])
+def test_gelu_tanh_rounding(ctx, std, lim):
+    """The 2-norm error of 0.5 v (1 + tanh(u)): where v > 0 holds the norm, 1 + tanh(u) is
+    rounded beside a sum near 2 (1.7e-8 of it, root mean square) and the product once
+    (2.5e-8), and neither is where tanh(u) is 1; 3.9e-8 with the rounding of u, 1 sigma.
+    A reciprocal of 1 + exp(-2u) rounds its sum beside 1 (4.2e-8, 3.3e-8 and 1.6e-8)."""
+    x = rnd(1 << 20, 62, std)
+    v = x.astype(np.float64)
+    ref = 0.5 * v * (1.0 + np.tanh(np.float32(0.7978845608028654).astype(np.float64)
+                                   * (v + np.float32(0.044715).astype(np.float64) * v ** 3)))
+    got = rt.GeluTanh(T(ctx, x)).numpy()
+    assert np.linalg.norm(got - ref) <= lim * np.linalg.norm(ref)
+
+
 def test_argmax_exact(ctx):
     rng = np.random.default_rng(70)
     for n in (1, 7, 50257, 1 << 20):
