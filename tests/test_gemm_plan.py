@@ -51,6 +51,17 @@ def test_value_shapes_reach_every_kernel():
     assert any(form(*s) == "128x1" and s[2] < 64 for s in T.EPILOGUES)
 
 
+@pytest.mark.parametrize("K", [32, 64, 256, 640, 768, 1024])
+def test_small_m_kernel_up_to_one_block_per_cu(K):
+    """Blocks of 32 rows by 48 columns, or 64 where N is no multiple of 48; above one a CU
+    the 64x64 tiles are faster at every K below 2048."""
+    for M, N in [(128, 3072), (160, 2304), (512, 768), (128, 4096), (256, 2048), (168, 768)]:
+        assert form(M, N, K) == "small", (M, N)
+    for M, N in [(129, 3072), (512, 3072), (192, 2304), (129, 4096), (257, 2048), (300, 2308)]:
+        assert form(M, N, K) != "small", (M, N)
+        assert form(M, N, K, tb=1) != "small", (M, N)
+
+
 def test_few_tiles_split_k():
     assert plan(64, 63, 1500)["splits"] == 7 and plan(64, 63, 575)["splits"] == 1
     assert plan(600, 256, 1000)["splits"] == 5  # 40 tiles
