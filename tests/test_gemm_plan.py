@@ -45,8 +45,8 @@ def test_value_shapes_reach_every_kernel():
     for shapes in (T.RANGES, T.MEETS):
         got = {form(*s, tb=tb) for s in shapes for tb in (0, 1)}
         assert {"small", "64x2", "128x1"} <= got
-    assert {form(M, N, 160, ta=ta, tb=tb) for ta, tb, M, N in T.INFINITIES} >= {
-        "small", "64x2", "128x1"}
+    got = {(form(M, N, K, ta=ta, tb=tb), tb) for ta, tb, M, N, K in T.INFINITIES}
+    assert got >= {("small", 0), ("small", 1), ("64x2", 0), ("128x1", 0), ("128x1", 1)}
     assert {form(*s) for s in T.EPILOGUES} >= {"64x2", "64x1", "128x1"}
     assert any(form(*s) == "128x1" and s[2] < 64 for s in T.EPILOGUES)
 
@@ -60,6 +60,14 @@ def test_small_m_kernel_up_to_one_block_per_cu(K):
     for M, N in [(129, 3072), (512, 3072), (192, 2304), (129, 4096), (257, 2048), (300, 2308)]:
         assert form(M, N, K) != "small", (M, N)
         assert form(M, N, K, tb=1) != "small", (M, N)
+
+
+def test_small_m_kernel_16_row_blocks_transposed():
+    """Above one block a CU, tiles for a short K with B transposed alone."""
+    for M, N in [(64, 2304), (64, 3072), (256, 768)]:
+        assert form(M, N, 256, tb=1) == form(M, N, 32, tb=1) == "64x2"
+        assert form(M, N, 260, tb=1) == form(M, N, 256) == form(M, N, 32) == "small"
+    assert form(64, 2048, 256, tb=1) == "small"  # 256 blocks
 
 
 def test_few_tiles_split_k():

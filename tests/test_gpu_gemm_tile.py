@@ -69,7 +69,8 @@ def test_gemm_tile_edges(ctx, ta, tb, M, N, K):
 # M <= 512 with whole float4 rows: every form of the small-M kernel (16x16,
 # 16x32, 16x48 over two blocks, 32x64, 32x48) and the tiles that replace it
 # from two or three rounds of blocks up
-SMALL = [(2, 4, 4), (33, 64, 60), (31, 768, 64), (17, 132, 68), (97, 772, 100), (130, 1540, 96),
+SMALL = [(2, 4, 4), (33, 64, 60), (127, 2304, 60), (120, 1732, 36), (31, 768, 64),
+         (64, 2304, 132), (17, 132, 68), (97, 772, 100), (130, 1540, 96),
          (130, 1732, 96), (128, 768, 3072), (100, 768, 2052), (127, 2304, 288),
          (255, 2304, 288), (129, 3072, 772), (300, 2308, 768), (259, 2308, 100), (130, 4100, 772),
          (512, 3072, 768), (131, 768, 2048)]
@@ -207,14 +208,15 @@ def test_gemm_zero_rows_that_stay_zero_or_not(ctx, M, N, K, ta):
     assert np.abs(got[10] - want).max() <= 2.0 ** -22 * np.abs(want).max()
 
 
-INFINITIES = [(0, 0, 777, 333), (1, 1, 777, 333), (0, 1, 500, 332), (0, 0, 2000, 2003),
-              (0, 1, 2000, 2003), (1, 0, 2000, 2003)]
+INFINITIES = [(0, 0, 777, 333, 160), (1, 1, 777, 333, 160), (0, 1, 500, 332, 160),
+              (0, 1, 500, 332, 288), (0, 0, 500, 332, 160), (0, 0, 2000, 2003, 160),
+              (0, 1, 2000, 2003, 160), (1, 0, 2000, 2003, 160)]
 
 
-@pytest.mark.parametrize("ta,tb,M,N", INFINITIES)
-def test_gemm_tile_infinities_and_nan(ctx, ta, tb, M, N):
-    """(N = 332 with 500 rows: the small-M kernel; 2000 rows: 128x128 tiles)"""
-    K = 160
+@pytest.mark.parametrize("ta,tb,M,N,K", INFINITIES)
+def test_gemm_tile_infinities_and_nan(ctx, ta, tb, M, N, K):
+    """(500 rows: the small-M kernel, with B transposed from K = 260; 2000 rows: 128x128
+    tiles)"""
     rng = np.random.default_rng(9)
     a = rng.standard_normal((M, K)).astype(np.float32)
     b = rng.standard_normal((K, N)).astype(np.float32)
