@@ -70,8 +70,8 @@ def test_gemm_tile_edges(ctx, ta, tb, M, N, K):
 # 16x32, 16x48 over two blocks, 32x64, 32x48) and the tiles that replace it
 # from two or three rounds of blocks up
 SMALL = [(2, 4, 4), (33, 64, 60), (127, 2304, 60), (120, 1732, 36), (31, 768, 64),
-         (64, 2304, 132), (17, 132, 68), (17, 132, 420), (97, 772, 100), (97, 772, 708), (130, 1540, 96),
-         (130, 1732, 96), (128, 768, 3072), (100, 768, 2052), (127, 2304, 288),
+         (64, 2304, 132), (17, 132, 68), (17, 132, 420), (97, 772, 100), (97, 772, 708),
+         (130, 1540, 96), (130, 1732, 96), (128, 768, 3072), (100, 768, 2052), (127, 2304, 288),
          (255, 2304, 288), (129, 3072, 772), (300, 2308, 768), (259, 2308, 100), (130, 4100, 772),
          (512, 3072, 768), (131, 768, 2048)]
 
@@ -233,6 +233,20 @@ def test_gemm_tile_infinities_and_nan(ctx, ta, tb, M, N, K):
     np.testing.assert_array_equal(got[inf], ref[inf])
     ok = np.isfinite(ref) & (np.abs(ref) < 1e30)
     assert np.abs(got[ok] - ref[ok]).max() <= 1e-3
+
+
+@pytest.mark.parametrize("tb", [0, 1])
+@pytest.mark.parametrize("K,lim", [(64, 8.7e-8), (128, 9.2e-8), (256, 1.0e-7)])
+def test_small_m_one_group_rounding(ctx, K, lim, tb):
+    """K up to 256 is eight sums of at most 32 products in the 16-row blocks: over half-zero
+    rows 8.0e-8, 8.5e-8 and 9.4e-8 in the 2-norm with exact operands, where pairs (rounded
+    at 2^-24 each) come to 9.4e-8, 9.9e-8 and 1.06e-7."""
+    for M, N in [(32, 768), (300, 300)]:
+        rng = np.random.default_rng(K + M)
+        a = np.maximum(rng.standard_normal((M, K)), 0).astype(np.float32)
+        b = (0.02 * rng.standard_normal((K, N))).astype(np.float32)
+        ref = a.astype(np.float64) @ b
+        assert np.linalg.norm(_run(ctx, a, b, 0, tb) - ref) <= lim * np.linalg.norm(ref)
 
 
 EPILOGUES = [(530, 70, 96), (4200, 1000, 96), (2000, 1990, 96), (1990, 2001, 40)]
