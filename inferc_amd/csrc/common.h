@@ -323,8 +323,8 @@ void gemm_qkv(inferc_hip_ctx* ctx, int64_t M, int64_t K, int64_t N, const float*
               int64_t ldy, const RowNorm* norm_a = nullptr);
 
 // Whether an unbatched, untransposed product with 16-byte aligned operands
-// (M x K times K x N, `slices` such products sharing A) takes the small-M
-// path, the one that supports RowNorm operands and stats_out.
+// (M x K times K x N, `slices` such products sharing A) runs the small-M
+// kernel, the one that supports RowNorm operands and stats_out.
 bool gemm_small_m_path(const inferc_hip_ctx* ctx, int64_t M, int64_t N, int64_t K,
                        int64_t slices);
 

@@ -2,8 +2,8 @@
 writes the row statistics of its output h, and the GEMMs that read the
 LayerNorm of h (A of FusedQKV, FusedMatMulAddGELU or FusedGemmEpilogue, the
 residual of a FusedGemmEpilogue) normalize h as they read it, so the LayerNorm kernel does
-not run. That holds while every product takes the small-M path (M <= 512);
-above it the LayerNorm kernel runs as before. Both against a float64
+not run. That holds while every product takes the small-M path (M <= 512, and at most
+one 32-row block a CU); above it the LayerNorm kernel runs as before. Both against a float64
 statement of the unfused graph (src/kernels/activation.cc:103-150 for the
 LayerNorm, fused_matmul_add_gelu.cc for the GELU epilogue), 1e-4."""
 from __future__ import annotations
@@ -13,7 +13,7 @@ import math
 import numpy as np
 import pytest
 
-from inferc_amd import rt
+from inferc_amd import lib as L, rt
 
 pytestmark = pytest.mark.gpu
 
@@ -24,7 +24,7 @@ def _w(rng, *shape, std=0.05):
     return (rng.standard_normal(shape) * std).astype(np.float32)
 
 
-def _graph(rng):
+def _graph(rng, H=H, F=F):
     """out-proj(+x0) -> LN1 -> {QKV, FFN-up -> FFN-down(+LN1), a plain
     projection} -> LN2 -> out-proj(+LN2) -> LN3. LN1 and LN2 are read by GEMMs
     only; LN3 is an output and stays a kernel."""
@@ -129,3 +129,36 @@ def test_two_layernorms_of_one_input_stay_kernels(ctx):
         got = ex.run(feeds, ["f", "z"])
         for nm in ("f", "z"):
             assert float(np.max(np.abs(got[nm] - ref[nm]))) <= 1e-4, nm
+
+
+@pytest.mark.parametrize("M,H,F,read", [
+    (256, 384, 1536, True),   # 256 blocks of 32x48 for FFN-up: one a CU
+    (288, 384, 1536, False),  # 288
+    (512, 256, 1024, True),   # 16 x 16 blocks of 32x64
+    (160, 768, 3072, False),  # 5 x 64
+])
+def test_layernorm_read_only_while_the_small_m_kernel_is_the_faster(ctx, M, H, F, read):
+    """Where a reader's product runs 64x64 tiles, the LayerNorm is a kernel of its own: its
+    readers' results are then the bits of LayerNorm and product one by one."""
+    rng = np.random.default_rng(M)
+    g, p = _graph(rng, H, F)
+    ex = rt.Executor(ctx, g)
+    feeds = {k: rng.standard_normal((M, H)).astype(np.float32) for k in ("x0", "a", "a2")}
+    got = ex.run(feeds, ["q", "z", "x3"])
+    ref = _reference(p, *(feeds[k].astype(np.float64) for k in ("x0", "a", "a2")))
+    for nm in got:
+        assert float(np.max(np.abs(got[nm] - ref[nm]))) <= 1e-4, nm
+    t = {k: rt.Tensor.from_numpy(ctx, v) for k, v in {**p, **feeds}.items()}
+    out = {k: rt.Tensor(ctx, (M, H), np.float32) for k in ("h1", "q", "k", "v")}
+
+    def ptr(*names):
+        return [(t | out)[n].ptr for n in names]
+
+    lib = L.load_library()
+    a, wo, bo, x0, h1 = ptr("a", "wo", "bo", "x0", "h1")
+    L.check(lib.inferc_hip_gemm_f32(ctx.handle, 0, 0, M, H, H, 1.0, a, H, wo, H, 1.0, bo, L.C_ROW,
+                                    0, x0, H, L.ACT_NONE, h1, H))
+    x1 = rt.LayerNorm(out["h1"], t["g1"], t["b1"], 1e-12)
+    L.check(lib.inferc_hip_fused_qkv_f32(ctx.handle, M, H, H, x1.ptr, *ptr(
+        "wq", "bq", "wk", "bk", "wv", "bv", "q", "k", "v")))
+    assert np.array_equal(got["q"], out["q"].numpy()) is not read
