@@ -65,9 +65,15 @@ def test_small_m_kernel_up_to_one_block_per_cu(K):
 def test_small_m_kernel_16_row_blocks_transposed():
     """Above one block a CU, tiles for a short K with B transposed alone."""
     for M, N in [(64, 2304), (64, 3072), (256, 768)]:
-        assert form(M, N, 256, tb=1) == form(M, N, 32, tb=1) == "64x2"
+        assert form(M, N, 256, tb=1) == "64x2" and form(M, N, 32, tb=1) == "64x1"
         assert form(M, N, 260, tb=1) == form(M, N, 256) == form(M, N, 32) == "small"
     assert form(64, 2048, 256, tb=1) == "small"  # 256 blocks
+
+
+def test_one_panel_has_one_group():
+    for M, N in [(516, 64), (600, 600), (204, 5903)]:
+        assert form(M, N, 32, ta=1) == form(M, N, 24, ta=1) == "64x1"
+        assert form(M, N, 33, ta=1) == "64x2"
 
 
 def test_few_tiles_split_k():

@@ -51,10 +51,11 @@ def _check(got, a, b):
 # M > 512 keeps the small-M kernel away; the tile forms' edges are 64 and 128
 EDGES_64 = [(513, 1, 1), (513, 65, 31), (576, 63, 32), (640, 129, 33), (515, 64, 63),
             (520, 68, 64), (519, 130, 65), (1000, 257, 96), (513, 384, 1536), (514, 131, 1601),
-            (4097, 1025, 68), (4100, 1100, 40), (70, 40001, 65), (40000, 66, 96)]
+            (4097, 1025, 68), (4100, 1100, 40), (70, 40001, 65), (40000, 66, 96),
+            (516, 64, 4), (600, 132, 12), (1000, 260, 28), (2600, 1200, 24)]
 EDGES_128 = [(5120, 1280, 128), (2000, 2000, 130), (1921, 2047, 1), (2047, 1921, 31),
              (2001, 1999, 45), (1990, 2011, 63), (1985, 1985, 64), (2033, 1987, 97),
-             (100, 50257, 40)]
+             (100, 50257, 40), (2000, 2000, 20)]
 
 
 @pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
