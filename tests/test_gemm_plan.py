@@ -70,6 +70,14 @@ def test_small_m_kernel_16_row_blocks_transposed():
     assert form(64, 2048, 256, tb=1) == "small"  # 256 blocks
 
 
+def test_long_k_transposed():
+    """Tiles above 128 rows, but up to K = 3072 not where 16x16 blocks take the product."""
+    for K in (2048, 3072):
+        assert form(200, 64, K, tb=1) == form(132, 4, K, tb=1) == form(200, 768, K) == "small"
+        assert form(128, 768, K, tb=1) == "small" and form(132, 256, K, tb=1) == "64x2"
+    assert form(200, 64, 3076, tb=1) == "64x2"
+
+
 def test_one_panel_has_one_group():
     for M, N in [(516, 64), (600, 600), (204, 5903)]:
         assert form(M, N, 32, ta=1) == form(M, N, 24, ta=1) == "64x1"

@@ -74,7 +74,7 @@ SMALL = [(2, 4, 4), (33, 64, 60), (127, 2304, 60), (120, 1732, 36), (31, 768, 64
          (64, 2304, 132), (17, 132, 68), (17, 132, 420), (97, 772, 100), (97, 772, 708),
          (130, 1540, 96), (130, 1732, 96), (128, 768, 3072), (100, 768, 2052), (127, 2304, 288),
          (255, 2304, 288), (129, 3072, 772), (300, 2308, 768), (259, 2308, 100), (130, 4100, 772),
-         (512, 3072, 768), (131, 768, 2048)]
+         (512, 3072, 768), (131, 768, 2048), (200, 60, 2052)]
 
 
 @pytest.mark.parametrize("tb", [0, 1])
