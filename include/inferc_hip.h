@@ -15,6 +15,18 @@
  *  - Device pointers are caller-owned unless a function says otherwise.
  *    Inputs are read-only; outputs must not alias inputs unless stated.
  *  - Matrices are row-major with leading dimensions counted in elements.
+ *
+ * Precision of the _f32 products and of attention. Dense products (gemm, matmul, fused QKV and
+ * FFN, the executor's and the decoder's prompt pass) accumulate in fp32. From K = 64 up (above
+ * 256 in the smallest tiles) they multiply each operand as a pair of fp16 numbers, 22 to 24 bits of it,
+ * so long as that loses less than K 2^-23 of the sum of |a| |b| of every output (twice the bound
+ * of an fp32 sum's rounding); where it could lose more, beside infinities and NaN, and where an
+ * output is a single product (a selection, which stays exact), the same kernel runs the fp32
+ * matrix instructions on the operands as they are. Error against 64 bits in the 2-norm over
+ * N(0, 1) x N(0, 0.02): 1.2e-7 to 1.5e-7 at K = 768, 1.3e-7 to 2.0e-7 at K = 3072, where the
+ * fp32 instructions give 1.9e-7 to 2.5e-7 and 1.9e-7 to 5.0e-7. Attention on large grids
+ * multiplies Q K^T as such pairs (loss below 2^-20 of a score) and the probabilities and V as
+ * three bf16 parts each, which hold all 24 bits. There is no reduced-precision mode.
  */
 #ifndef INFERC_HIP_H_
 #define INFERC_HIP_H_
