@@ -3,6 +3,7 @@ the GPU tests run the kernels they are there for, and the grid of the widest pro
 from __future__ import annotations
 
 import ctypes as C
+import random
 
 import pytest
 
@@ -89,6 +90,22 @@ def test_few_tiles_split_k():
     assert plan(600, 256, 1000)["splits"] == 5  # 40 tiles
     assert plan(700, 700, 768)["splits"] == 1  # 121 tiles: no CU is idle
     assert plan(512, 768, 3072, tb=1)["splits"] == 4
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0)])
+def test_partial_sums_fit_the_scratch(ta, tb):
+    """A context starts with 16 MiB of workspace, and the allocation-free entry point has no
+    more: the partial sums of any product fit, so that none is refused under capture."""
+    rng = random.Random(ta + 2 * tb)
+    for _ in range(4000):
+        M, N, K = (int(round(2 ** rng.uniform(0, top))) for top in (13, 13, 15))
+        if rng.random() < 0.5:
+            M, N, K = (max(4, x // 4 * 4) for x in (M, N, K))
+        p = plan(M, N, K, ta=ta, tb=tb)
+        if p["groups"] == 0:  # whole tiles, one for each of the z blocks
+            M, N = -(-M // p["rows"]) * p["rows"], -(-N // p["cols"]) * p["cols"]
+        if p["splits"] > 1:
+            assert 4 * p["splits"] * M * N <= 16 << 20, (M, N, K, p)
 
 
 @pytest.mark.parametrize("M,N", [(1, 2 ** 31 - 65), (64, 2 ** 30 + 1), (100, 2 ** 31 - 65),
